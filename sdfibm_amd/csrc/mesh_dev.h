@@ -330,13 +330,14 @@ __device__ inline R cell_fraction(const MeshDev& m, const SolidK& K, int i, int 
             box_corner_phi(m, K, i, j, k, h, lc);
         const double z0 = m.zs[k], z1 = m.zs[k + 1];
         const float az = (float)((0.0 - z0) / (z1 - z0));
-        return box_fraction<float, PL>(h, i == 0, j == 0, k == 0, m.two_d != 0, az);
+        return box_fraction<float, PL>(h, i == 0, j == 0, k == 0, m.two_d != 0, az, has_poles(K.shape));
     } else if constexpr (MK == MK_RECT) {
         if (PL && K.shape == SDFIBM_SHAPE_PLANE) return fraction_of_cell<R, MK>(m, K, i, j, k);
         Phi8<double> h;
         box_corner_phi64(m, K, i, j, k, h);
         const double z0 = m.zs[k], z1 = m.zs[k + 1];
-        return box_fraction<double>(h, i == 0, j == 0, k == 0, m.two_d != 0, (0.0 - z0) / (z1 - z0));
+        return box_fraction<double>(h, i == 0, j == 0, k == 0, m.two_d != 0, (0.0 - z0) / (z1 - z0),
+                                    has_poles(K.shape));
     } else {
         return fraction_of_cell<R, MK>(m, K, i, j, k);
     }

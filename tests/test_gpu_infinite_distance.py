@@ -86,3 +86,31 @@ def test_ellipsoid_taken_off_structured(size):
     for (ca, fa), (cb, fb) in zip(a, b):
         np.testing.assert_array_equal(ca, cb)
         assert np.max(np.abs(fa - fb), initial=0.0) <= TOL["fp32"]
+
+
+BALL = [("ellipsoid", "union", (1.0, 0.9, 1.1))]
+FLAT_VOIDS = ([("box", "union", (1.3, 1.3, 1.3)), ("ellipsoid", "difference", (0.35, 1.25, 1.2))],
+              [("sphere", "union", (1.5,)), ("ellipsoid", "difference", (1.25, 0.35, 1.2))],
+              [("sphere", "union", (1.5,)), ("ellipsoid", "difference", (1.25, 1.2, 0.35))])
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("size", [0.6, 0.95, 1.2, 1.45, 1.7, 2.3])
+@pytest.mark.parametrize("which", ["ellipse2d", "ellipse3d", "csg"])
+def test_centre_on_a_vertex(which, size, prec):
+    """A cut cell with a corner at -inf: its edges to inside corners lie inside."""
+    flat = which == "ellipse2d"
+    _against_oracle(*_scene(BALL if which == "csg" else S.ELLIPSE, size, flat), prec, flat)
+
+
+@pytest.mark.parametrize("size", [0.6, 0.95, 1.2])
+def test_ellipsoid_centre_on_a_vertex_fp32(size):
+    _against_oracle(*_scene(S.ELLIPSOID, size), "fp32")
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("size", [0.6, 0.8, 0.95, 1.2, 1.7])
+@pytest.mark.parametrize("void", range(len(FLAT_VOIDS)))
+def test_faces_outside_with_a_corner_at_infinity(void, size, prec):
+    """A face of a cut cell wholly outside whose first corner is the void's centre has no area inside."""
+    _against_oracle(*_scene(FLAT_VOIDS[void], size), prec)
