@@ -114,3 +114,12 @@ def test_ellipsoid_centre_on_a_vertex_fp32(size):
 def test_faces_outside_with_a_corner_at_infinity(void, size, prec):
     """A face of a cut cell wholly outside whose first corner is the void's centre has no area inside."""
     _against_oracle(*_scene(FLAT_VOIDS[void], size), prec)
+
+
+@pytest.mark.parametrize("axes", [(0.6, 1.5, 1.6), (1.5, 0.6, 1.6), (1.6, 1.5, 0.6), (0.9, 0.8, 2.2), (1.2, 1.1, 1.0)])
+def test_ellipsoid_centre_on_a_vertex_fp64(axes):
+    """The reciprocal root of the zero squared length at the centre is infinite, not NaN: an edge from
+    there to outside has no fraction."""
+    mesh, sol, _ = _scene(S.ELLIPSOID, 1.0)
+    sol["prm"][:, :3] = np.array(axes) * H
+    _against_oracle(mesh, sol, None, "fp64")
