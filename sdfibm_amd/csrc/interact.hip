@@ -2819,6 +2819,12 @@ int setup_mesh(sdfibm_ctx* c, const sdfibm_mesh_desc* d) {
 template <class R, int MK>
 int interact_impl(sdfibm_ctx* c, double dt, const StepEnd& end) {
     const int r = launch_step<R, MK>(c, dt, end);
+    if (r != 0 && !end.graph) {
+        // given up between the fork and the join: the second stream may still bin and label big
+        // tiles, and the next step's reset and setup are ordered after the main stream only
+        (void)hipStreamSynchronize(c->aux);
+        (void)hipStreamSynchronize(c->stream);
+    }
     HIPCHK(c, hipGetLastError());
     if (r == -1) return fail(c, SDFIBM_ERR_HIP, "plane component pass: HIP copy/synchronize failed");
     if (r == -2) return fail(c, SDFIBM_ERR_CAPACITY, "plane component labelling did not converge");
