@@ -4263,8 +4263,9 @@ int sdfibm_interact(sdfibm_ctx* c, double time, double dt, double* ft) {
         }
         if ((rc = step())) return rc;
     }
-    if (end.host_ft && c->ns < kFtBeside) std::memcpy(ft, c->h_ft, c->ns * 48);
-    if (end.host_ft && c->ns >= kFtBeside && !flags)
+    if (end.host_ft && (c->ns < kFtBeside || flags))  // beside the field pass: copied above if no flag was raised
+        std::memcpy(ft, c->h_ft, c->ns * 48);
+    else if (end.host_ft)
         for (const int sp : c->h_planes) std::memcpy(ft + 6LL * sp, c->h_ft + 6LL * sp, 48);
     float ms[5] = {0, 0, 0, 0, 0};
     if (c->phase_timing) {
