@@ -3134,29 +3134,41 @@ int poly_setup(sdfibm_ctx* c, const sdfibm_polymesh_desc* d) {
     for (long long k = 0; k < nC; ++k)
         if (!(vp[k] > 0)) return fail(c, SDFIBM_ERR_MESH, "cell " + std::to_string(k) + " has no positive volume");
     // bins: a uniform grid over the cell centres' box, about 4 cells per bin; each bin's box
-    // holds its cells' point boxes
+    // holds its cells' point boxes.  An axis along which the centres spread by less than a
+    // bin's side takes one bin (a mesh one cell thick, whose centres differ by rounding, had
+    // 4096 x 4096 bins, 0.8 GB, and a search for a nearest cell over them took seconds)
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     for (long long k = 0; k < nC; ++k)
         for (int e = 0; e < 3; ++e) {
             lo[e] = std::min(lo[e], ccp[3 * k + e]);
             hi[e] = std::max(hi[e], ccp[3 * k + e]);
         }
-    double ext[3], vol_box = 1.0;
-    int dims = 0;
+    double ext[3], side = 1.0;
+    bool on[3];
     for (int e = 0; e < 3; ++e) {
         ext[e] = hi[e] - lo[e];
-        if (ext[e] > 0) {
-            vol_box *= ext[e];
-            ++dims;
-        }
+        on[e] = ext[e] > 0;
     }
     const double want = std::max(1.0, (double)nC / 4.0);
-    const double side = dims > 0 ? std::pow(vol_box / want, 1.0 / dims) : 1.0;
+    for (;;) {
+        double vol_box = 1.0;
+        int dims = 0, thin = -1;
+        for (int e = 0; e < 3; ++e)
+            if (on[e]) {
+                vol_box *= ext[e];
+                ++dims;
+                if (thin < 0 || ext[e] < ext[thin]) thin = e;
+            }
+        if (dims == 0) break;
+        side = std::pow(vol_box / want, 1.0 / dims);
+        if (ext[thin] >= side) break;
+        on[thin] = false;
+    }
     PolyDev& P = c->pm;
     long long nb = 1;
     for (int e = 0; e < 3; ++e) {
-        P.bn[e] = ext[e] > 0 ? (int)std::max(1.0, std::min(4096.0, std::floor(ext[e] / side))) : 1;
-        P.bw[e] = ext[e] > 0 ? ext[e] / P.bn[e] : 1.0;
+        P.bn[e] = on[e] ? (int)std::max(1.0, std::min(4096.0, std::floor(ext[e] / side))) : 1;
+        P.bw[e] = on[e] ? ext[e] / P.bn[e] : std::max(ext[e], side);
         P.binv[e] = 1.0 / P.bw[e];
         P.blo[e] = lo[e];
         nb *= P.bn[e];
@@ -3205,7 +3217,7 @@ int poly_setup(sdfibm_ctx* c, const sdfibm_polymesh_desc* d) {
             bbox[6 * b + 3 + e] = std::max(bbox[6 * b + 3 + e], ch[e]);
             const double blo = P.blo[e] + ijk[e] * P.bw[e], bhi = blo + P.bw[e];
             const double over = std::max(blo - cl[e], ch[e] - bhi);
-            if (over > 0) reach = std::max(reach, (int)std::ceil(over * P.binv[e]));
+            if (over > 0 && P.bn[e] > 1) reach = std::max(reach, (int)std::ceil(over * P.binv[e]));
         }
     }
     c->poly_reach = std::min(reach, 4096);

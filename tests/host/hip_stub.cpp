@@ -3,6 +3,7 @@
 // what a call leaves behind on its streams without a GPU.
 //   stub_fail_copies(n)  the n-th hipMemcpyAsync from now on fails (0: none)
 //   stub_busy()          launches the host has not waited for, over all streams
+//   stub_bytes()         device memory asked for so far
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -22,6 +23,7 @@ struct Config {
     void* stream;
 } config;
 int fail_in = 0;
+long long asked = 0;
 constexpr int kError = 999;  // hipErrorUnknown
 
 void join(Clock& a, const Clock& b) {
@@ -34,6 +36,7 @@ void* handle() { return std::calloc(1, 8); }
 
 extern "C" {
 void stub_fail_copies(int n) { fail_in = n; }
+long long stub_bytes() { return asked; }
 long long stub_busy() {
     long long n = 0;
     for (auto& s : streams) n += s.second[s.first] - done[s.first];
@@ -90,7 +93,10 @@ int hipEventElapsedTime(float* ms, void*, void*) {
     return 0;
 }
 
-int hipMalloc(void** p, size_t n) { return alloc(p, n); }
+int hipMalloc(void** p, size_t n) {
+    asked += (long long)n;
+    return alloc(p, n);
+}
 int hipFree(void* p) {
     std::free(p);
     return 0;
