@@ -4866,10 +4866,16 @@ int sdfibm_pair_counts(sdfibm_ctx* c, int64_t* out) {
     if (ns == 0) return SDFIBM_OK;
     std::vector<int2> nc(ns);
     HIPCHK(c, hipMemcpy(nc.data(), c->d_ncand, ns * sizeof(int2), hipMemcpyDeviceToHost));
-    std::vector<char> is_plane(ns, 0);
-    for (int p : c->h_planes) is_plane[p] = 1;
+    std::vector<char> skip(ns, 0);  // planes, and solids without a tile, whose counts no kernel writes
+    for (int p : c->h_planes) skip[p] = 1;
+    if (c->kind != SDFIBM_MESH_POLY) {
+        std::vector<TileInfo> T(ns);
+        HIPCHK(c, hipMemcpy(T.data(), c->d_T, ns * sizeof(TileInfo), hipMemcpyDeviceToHost));
+        for (long long s = 0; s < ns; ++s)
+            if (T[s].cls == TC_EMPTY) skip[s] = 1;
+    }
     for (long long s = 0; s < ns; ++s)
-        if (!is_plane[s]) {
+        if (!skip[s]) {
             out[0] += nc[s].x;
             out[1] += nc[s].y;
         }
