@@ -4,8 +4,9 @@
 ``sdfibm_amd/libsdfibm_hip.so`` with hipcc.  Flags:
 
 * ``--offload-arch=gfx950``: MI355X only;
-* ``-ffp-contract=off``: no fused multiply-add, so the FP64 inside tests and
-  fractions round exactly like the CPU (candidate lists bit-identical);
+* ``-ffp-contract=off``: no fused multiply-add but where the source asks for one, so the
+  FP64 inside tests round exactly like the CPU (candidate lists bit-identical; FP64
+  fractions agree to 1e-12);
 * ``-Xclang -target-feature -Xclang -packed-fp32-ops``: no packed FP32 math.
 """
 from __future__ import annotations

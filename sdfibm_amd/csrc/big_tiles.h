@@ -46,7 +46,7 @@
 //                   -> force/torque
 #pragma once
 
-constexpr int kBigPer = 16;                  // big solids per thread of the one-workgroup scans
+constexpr int kBigPer = 16;                  // big solids per thread of k_big_chunks
 constexpr int kBigMaxSolids = 1024 * kBigPer;  // big tiles per step (SDFIBM_ERR_CAPACITY beyond)
 constexpr int kBigChunk = 1024;      // default candidate entries per chunk of k_big_force (the autotuner's choice)
 constexpr int kBigUPB = 256;         // units, and vertex words, per block (a thread each)

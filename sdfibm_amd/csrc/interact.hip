@@ -111,9 +111,10 @@ __device__ inline R code_none() {
     return R(__builtin_nan(""));
 }
 
-// q = a / b, r = a % b for 0 <= a < 2^22 and 1 <= b < 2^12, rb = 1.0f / b: the
-// truncated float product is within one of the quotient (relative error below
-// 2^-23 on a value below 2^22); one step corrects it.
+// q = a / b, r = a % b for 0 <= a < 2^22 and any b >= 1, rb = 1.0f / b: a is exact
+// in a float, the reciprocal and the product are each rounded once, so the product
+// is off the quotient a / b < 2^22 by less than 2^22 * 2^-23 = 1/2 whatever b is; its
+// integer part is within one of the quotient and one step corrects it.
 __device__ inline void divmod_small(int a, int b, float rb, int& q, int& r) {
     q = (int)((float)a * rb);
     r = a - q * b;
@@ -161,17 +162,6 @@ __host__ __device__ inline int tile_queue(int cls) {
     return cls == TC_SMALL ? 0 : (cls == TC_MEDIUM ? 1 : (cls == TC_BIG ? 4 : -1));
 }
 
-// The tiles' code and list offsets: one atomic per wave on the step's running
-// total (a bump allocation; the layout does not depend on the order, every tile
-// is addressed through its own offset), the wave's tiles in lane order.  On a
-// rectilinear mesh of up to kSetupStage vertex coordinates the three coordinate
-// arrays are staged in LDS first (dynamic LDS of setup_lds_bytes): each lane's
-// tile bounds and nearest cell are searches whose probes depend on each other,
-// served from LDS instead of memory.  The staging loop is a chain of loads too:
-// 256 threads, four loads in flight each (with 64 threads it was half of the
-// kernel's time: 12 us for 14 solids on a 200x200 mesh).
-// classes: bits of the tile classes whose kernels are launched (kClass*); a tile
-// of another class is flagged EF_TILE and the solids are classified again.
 // What the field pass needs of a solid, one cache line (its tile record and motion lie
 // in five lines of TileInfo and SolidK: 97 us of the field pass of 90,050 solids,
 // against 45 and 3 us more in k_setup): its tile (no layers where it
@@ -193,6 +183,18 @@ __host__ inline size_t setup_lds_bytes(const MeshDev& m, int mk) {
     return mk == MK_RECT && n <= kSetupStage ? (size_t)n * sizeof(double) : 0;
 }
 
+// Shape constants, tile, seed and field record of every solid, a thread each.
+// The tiles' code and list offsets: one atomic per wave on the step's running
+// total (a bump allocation; the layout does not depend on the order, every tile
+// is addressed through its own offset), the wave's tiles in lane order.  On a
+// rectilinear mesh of up to kSetupStage vertex coordinates the three coordinate
+// arrays are staged in LDS first (dynamic LDS of setup_lds_bytes): each lane's
+// tile bounds and nearest cell are searches whose probes depend on each other,
+// served from LDS instead of memory.  The staging loop is a chain of loads too:
+// 256 threads, four loads in flight each (with 64 threads it was half of the
+// kernel's time: 12 us for 14 solids on a 200x200 mesh).
+// classes: bits of the tile classes whose kernels are launched (kClass*); a tile
+// of another class is flagged EF_TILE and the solids are classified again.
 template <int MK>
 __global__ void __launch_bounds__(kSetupThreads) k_setup(const sdfibm_solid* __restrict__ in, int ns, MeshDev m, SolidK* __restrict__ K,
                         TileInfo* __restrict__ T, FieldRec* __restrict__ frec, long long* __restrict__ total,
@@ -2453,7 +2455,8 @@ void launch_big(sdfibm_ctx* c, double dt, hipStream_t st) {
 // Solids from which the force and torque are handed over beside the field pass, and
 // copied to the caller while it runs.  It saves the copies (90,050 solids: k_step_end
 // 82 -> 4 us and 130 us of the host, a step 1,450 -> 1,296 us) and costs two events and
-// a launch (14 solids: a step 78 -> 99 us); 10,000 solids take 436 us either way.
+// a launch (14 solids: a step 78 -> 99 us); 10,000 solids take 436 us either way.  At the
+// line it gains a little: 16,383 and 16,384 small spheres on 192^3 cells 174 and 168 us.
 constexpr int kFtBeside = 16384;
 
 // How a step ends: captured into a HIP graph (its error flags go into the sticky
@@ -4111,7 +4114,9 @@ int classify_solids(sdfibm_ctx* c, const sdfibm_solid* solids, int64_t n) {
     c->cell_set = cell_set_of(solids, n);
     // one wave per tiny or small tile only where there are waves enough to fill the chip: below
     // that a solid's own chain of rounds is what takes the time (14 discs of 600 cells: 31 us a
-    // wave each in the cut-cell pass, 13 us with 256 threads)
+    // wave each in the cut-cell pass, 13 us with 256 threads).  At the line the steps are close,
+    // the one-wave side the shorter: 2,047 and 2,048 spheres of 2-4 cells on 128^3 cells 77 and
+    // 72 us (FP64 91 and 81), of 4-7 cells 88 and 87; discs of radius 3, 83 and 75 us
     const long long fill = 8LL * c->n_cu;
     c->small_tiles = n_tiles >= fill && tile_sum < 512 * n_tiles;
     if (n_tiny >= fill) {
