@@ -151,8 +151,9 @@ __device__ inline R sdf_fast(const SolidK& K, d3 p) {
 
 // Volume fraction of cell (i,j,k) (calcCellVolume / V) from its 8 corner signed
 // distances; phi_at(di, dj, dk) returns the distance at vertex (i+di, j+dj, k+dk).
+// poles: the solid's distance is infinite somewhere.
 template <class R, int MK, class PhiAt>
-__device__ inline R fraction_with_phi(const MeshDev& m, int i, int j, int k, PhiAt phi_at) {
+__device__ inline R fraction_with_phi(const MeshDev& m, int i, int j, int k, bool poles, PhiAt phi_at) {
     const d3 w0 = vertex_pos<MK>(m, i, j, k);
     Hex8<R> h;
     auto vtx = [&](int di, int dj, int dk, r3<R>& p, R& f) {
@@ -168,6 +169,7 @@ __device__ inline R fraction_with_phi(const MeshDev& m, int i, int j, int k, Phi
     vtx(1, 0, 1, h.p5, h.f5);
     vtx(0, 1, 1, h.p6, h.f6);
     vtx(1, 1, 1, h.p7, h.f7);
+    if (poles && infinite_corner<R>(h)) finite_corners<R>(h);
     const bool bnd[3] = {i == 0, j == 0, k == 0};
     const R V = R(cell_volume<MK>(m, i, j, k));
     return hex_fraction<R>(h, [&](int slot, r3<R>& fc, r3<R>& sf) { hex_face<R, MK>(m, i, j, k, w0, slot, fc, sf); },
@@ -177,7 +179,7 @@ __device__ inline R fraction_with_phi(const MeshDev& m, int i, int j, int k, Phi
 // Volume fraction of cell (i,j,k) inside solid K, corner distances evaluated here.
 template <class R, int MK>
 __device__ inline R fraction_of_cell(const MeshDev& m, const SolidK& K, int i, int j, int k) {
-    return fraction_with_phi<R, MK>(m, i, j, k, [&](int, int, int, d3 w) { return sdf_fast<R>(K, w); });
+    return fraction_with_phi<R, MK>(m, i, j, k, has_poles(K.shape), [&](int, int, int, d3 w) { return sdf_fast<R>(K, w); });
 }
 
 // Corner signed distances of box cell (i,j,k) of a rectilinear mesh in FP32

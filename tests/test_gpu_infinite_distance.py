@@ -21,15 +21,18 @@ H = 1.0 / 8
 TOL = {"fp64": 1e-12, "fp32": 1e-6}
 
 
-def _scene(shape, size, flat=False):
+def _scene(shape, size, flat=False, jitter=0.0):
     """One solid of `size` cells (a shape id, or CSG primitives in units of `size`) on each of some
     vertices of a 24 x 20 x 16 (x 1) mesh: mesh, solids, CSG table."""
     n = (24, 20, 1) if flat else (24, 20, 16)
-    mesh = M.uniform_box(n, (0, 0, -0.5 if flat else 0), (n[0] * H, n[1] * H, 0.5 if flat else n[2] * H))
+    box = (0, 0, -0.5 if flat else 0), (n[0] * H, n[1] * H, 0.5 if flat else n[2] * H)
+    mesh = M.jittered_box(n, *box, jitter, 3) if jitter else M.uniform_box(n, *box)
     g = np.meshgrid((0, 6, 12, 18, 24), (0, 7, 13, 20), (0,) if flat else (0, 8, 16), indexing="ij")
     at = np.stack(g, -1).reshape(-1, 3)
     sol = S.make_solids(len(at))
-    sol["center"] = at * H
+    sol["center"] = np.asarray(mesh.points)[at[:, 0] + (n[0] + 1) * (at[:, 1] + (n[1] + 1) * at[:, 2])]
+    if flat:
+        sol["center"][:, 2] = 0.0
     table = None
     if isinstance(shape, int):
         sol["shape"] = shape
@@ -52,13 +55,13 @@ def _lists(mesh, sol, table, prec, flat=False, structured=False):
         return [c.candidates(s)[1:] for s in range(sol.size)]
 
 
-def _against_oracle(mesh, sol, table, prec, flat=False, poly=False):
+def _against_oracle(mesh, sol, table, prec, flat=False, poly=False, structured=False):
     pm = mesh.to_polymesh()
     if table is not None:
         oracle.set_csg(np.atleast_1d(table))
     r = oracle.OracleMesh(pm).interact(sol, np.ones((mesh.n_cells, 3)), two_d=flat, rho_f=1.0, dt=1e-3,
                                        capture=True, capacity=40 * mesh.n_cells)
-    got = _lists(pm if poly else mesh, sol, table, prec, flat)
+    got = _lists(pm if poly else mesh, sol, table, prec, flat, structured)
     worst = 0.0
     for s, (_, cells, alpha) in enumerate(split_candidates(r, sol.size)):
         ref = {int(c): a for c, a in zip(cells, alpha) if np.isfinite(a)}
@@ -123,3 +126,15 @@ def test_ellipsoid_centre_on_a_vertex_fp64(axes):
     mesh, sol, _ = _scene(S.ELLIPSOID, 1.0)
     sol["prm"][:, :3] = np.array(axes) * H
     _against_oracle(mesh, sol, None, "fp64")
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("jitter", [0.0, 0.15])
+@pytest.mark.parametrize("size", [0.6, 0.95, 1.2, 1.7])
+@pytest.mark.parametrize("which", ["ellipse2d", "ellipsoid", "csg", "void0", "void1", "void2"])
+def test_general_hexahedra(which, size, jitter, prec):
+    """Cells of eight points that are not boxes: the corners the cell's apex does not take have no weight."""
+    flat = which == "ellipse2d"
+    shape = FLAT_VOIDS[int(which[-1])] if which.startswith("void") else \
+        dict(ellipse2d=S.ELLIPSE, ellipsoid=S.ELLIPSOID, csg=BALL)[which]
+    _against_oracle(*_scene(shape, size, flat, 0.0 if flat else jitter), prec, flat, structured=True)
